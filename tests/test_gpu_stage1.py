@@ -232,3 +232,35 @@ def test_key_halves_far_apart(split, dev):
         k[cu_k[b] + split:cu_k[b + 1]] *= 12.0
     d["k"] = k.to(torch.bfloat16)
     _check(d, _run(d, dev))
+
+
+@pytest.mark.parametrize("std", [1.0, 2.8, 4.2, 7.0])
+@pytest.mark.parametrize("lk", [511, 130])
+def test_small_scores_of_short_rows(lk, std, dev):
+    # Every score, also those far below the row's largest, against 64 bits.
+    # The kernel keeps a head's exponentials as truncated f16 against its max
+    # over the first 16 keys, or the row's max where a head's sum passes 65472:
+    # each is off by 2^-10 of itself or, below 2^-14 (subnormal), by 2^-24; the
+    # sums by 2^-10 at most, the f16 weights 1 / sum by 2^-11; exponents of
+    # |x| < 64 in fp32 by 2^-18 and the fp32 products behind them, 2^-14 in all.
+    T, G, Hkv = 256, 16, 2
+    g = torch.Generator(device=dev).manual_seed(int(10 * std) + lk)
+    q = torch.randn(T, G * Hkv, 128, generator=g, device=dev).to(torch.bfloat16)
+    k = (std * torch.randn(lk, Hkv, 128, generator=g, device=dev)).to(torch.bfloat16)
+    cu_q = torch.tensor([0, T], dtype=torch.int32, device=dev)
+    cu_k = torch.tensor([0, lk], dtype=torch.int32, device=dev)
+    out = infllmv2_attn_stage1(q, k, None, cu_q, cu_k, max_seqlen_k=lk, causal=False)
+    for h in range(Hkv):
+        x = torch.mm(q[:, G * h:G * h + G].double().reshape(T * G, 128),
+                     k[:, h].double().t().contiguous()).reshape(T, G, lk) * 128 ** -0.5
+        top = x.amax(-1, keepdim=True)
+        s_top = (x - top).exp().sum(-1)
+        s_ref = s_top * (top - x[:, :, :16].amax(-1, keepdim=True)).squeeze(-1).exp()
+        exact = ((x - top).exp() / s_top[..., None]).sum(1)
+        fast, slow = (1 / s_ref).sum(1), (1 / s_top).sum(1)
+        worst = s_ref.amax(1)
+        redone = worst > 65472 * (1 - 2 ** -9)  # near the line: the larger of the two bounds
+        unit = torch.where(redone, torch.maximum(fast, slow), fast)[:, None]
+        err = (out[h, :, :lk].double() - exact).abs()
+        bound = (2 ** -9 + 2 ** -11 + 2 ** -14) * exact + 2 ** -24 * (1 + 2 ** -9) * unit
+        assert bool((err <= bound).all()), float((err / bound).max())
