@@ -354,3 +354,38 @@ def test_two_rows_a_wave(T, B, order, dev):
         two = sparse_paged_attention(**pd, out_dtype=torch.float32)
         assert torch.equal(one.nan_to_num(nan=-7.0), two.nan_to_num(nan=-7.0))
         assert v_inf or torch.equal(two.cpu(), got)
+
+
+# One instance of the kernel each: rows shared by four waves, one row a wave,
+# two rows a wave, and the slot-table forms of the first two.
+@pytest.mark.parametrize("T,Hkv,B,slots", [(9, 2, 3, False), (9, 2, 3, True), (600, 2, 2, False),
+                                           (600, 2, 2, True), (1030, 4, 3, False)])
+def test_infinite_scores(T, Hkv, B, slots, dev):
+    # A key whose score is -inf has weight 0; a token whose every attended
+    # score is -inf has no softmax (NaN), and one that attends nothing is 0.
+    # The queries are positive in dim 0, where some keys hold -inf, but for one
+    # head of token 1, whose scores are +inf there: NaN, as inf - inf.
+    p = _problem(1200 + T, T=T, Hkv=Hkv, K=3, B=B, n_blocks=24, L=64 * 24, neg=0.2)
+    p["topk_idx"][:, 1] = torch.tensor([0, 1, 2], dtype=torch.int32)
+    p["token_pos_in_bs"][1] = 192
+    q = p["query"].view(T, Hkv, 16, 128)
+    q[..., 0] = q[..., 0].abs() + 0.5
+    q[1, :, 3, 0] = -1.0
+    rows = p["key_cache"].view(-1, 128)
+    rows[::3, 0] = float("-inf")
+    # Tokens 2 and 3 select one block each, whose every key holds -inf; token
+    # 3 attends 5 of its keys.  Token 4 attends nothing.
+    p["key_cache"][5, :, :, 0] = float("-inf")
+    p["topk_idx"][:, 2:4] = -1
+    p["topk_idx"][:, 2:4, 1] = 7
+    p["token_to_bs"][:6] = 0
+    p["block_table"][0, 7 * 64:8 * 64] = 5 * 64 + torch.arange(64, dtype=torch.int32)
+    p["seqlen_q"][0] = 64 * 24
+    p["token_pos_in_bs"][2:5] = torch.tensor([64 * 24, 7 * 64 + 5, 0], dtype=torch.int32)
+    exp = oracle_attn(**p)
+    assert torch.isnan(exp[2:4]).all() and not torch.isnan(exp[5:]).all() and (exp[4] == 0).all()
+    pd = {k: (v.to(dev) if isinstance(v, torch.Tensor) else v) for k, v in p.items()}
+    st = get_block_table(pd["topk_idx"], pd["block_table"], pd["token_to_bs"],
+                         pd["token_pos_in_bs"], pd["seqlen_q"], head_group=Hkv) if slots else None
+    got = sparse_paged_attention(**pd, slots=st, out_dtype=torch.float32).cpu()
+    torch.testing.assert_close(got, exp, atol=ATOL, rtol=RTOL, equal_nan=True)

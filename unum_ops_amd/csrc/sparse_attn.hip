@@ -49,6 +49,10 @@
 //     2^-15);
 //   * the running max moves only when a half's max exceeds it by more than
 //     8 (log2 units), so the O^T rescale is rare; exponentials stay <= 2^8.
+//     It starts at the lowest float, not at -inf, so a half of -inf scores
+//     adds zeros; a sum that is still zero at the end of a row that attended
+//     a key is a softmax over -inf alone: NaN, where a row that attended
+//     nothing is 0.
 #include <type_traits>
 
 #include "common.h"
@@ -532,10 +536,11 @@ __global__ __launch_bounds__(kWave* kSplit, 2) void sparse_attn_kernel(SaArgs a)
         acc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[u][cc], qf[kR][cc], acc[u], 0, 0, 0);
     float x[8] = {acc[0].x, acc[0].y, acc[0].z, acc[0].w, acc[1].x, acc[1].y, acc[1].z, acc[1].w};
     const bool whole = ok == 0x00FF00FF00FF00FFull;  // wave-uniform
+    const uint64_t mine = ok >> g;
+    auto attended = [&](int i) { return ((mine >> (16 * (i & 3) + 4 * (i >> 2))) & 1) != 0; };
     if (!whole) {
-      const uint64_t mine = ok >> g;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) x[i] = (mine >> (16 * (i & 3) + 4 * (i >> 2))) & 1 ? x[i] : -INFINITY;
+      for (int i = 0; i < 8; ++i) x[i] = attended(i) ? x[i] : -INFINITY;
     }
     float mx = fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), fmaxf(fmaxf(x[4], x[5]), fmaxf(x[6], x[7])));
     mx = sa_max_x32(sa_max_x16(mx)) * c;
@@ -555,9 +560,9 @@ __global__ __launch_bounds__(kWave* kSplit, 2) void sparse_attn_kernel(SaArgs a)
     float p[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) p[i] = __builtin_amdgcn_exp2f(fmaf(x[i], c, -m_run[kR]));
-    if (!whole) {  // a scale of zero times -inf is no -inf
+    if (!whole) {  // by the mask: a scale of zero times -inf is no -inf
 #pragma unroll
-      for (int i = 0; i < 8; ++i) p[i] = x[i] == -INFINITY ? 0.f : p[i];
+      for (int i = 0; i < 8; ++i) p[i] = attended(i) ? p[i] : 0.f;
     }
     l_run[kR] += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
     // P^T as two bf16 terms: hi = P truncated to bf16, lo = the exact residual
@@ -589,8 +594,10 @@ __global__ __launch_bounds__(kWave* kSplit, 2) void sparse_attn_kernel(SaArgs a)
           __builtin_bit_cast(bf16x8, __builtin_shufflevector(vf[dt][0], vf[dt][1], 0, 1, 2, 3, 4, 5, 6, 7)),
           __builtin_bit_cast(bf16x8, pl), o[kR][dt], 0, 0, 0);
   };
+  uint32_t seen = 0;  // the rows that attended a key (wave-uniform)
   auto compute = [&](uint64_t ok, uint32_t who) __attribute__((always_inline)) {
     if (ok == 0) return;
+    seen |= who;
     if (kRows == 1 || (who & 1)) compute_row(std::integral_constant<int, 0>{}, ok);
     if constexpr (kRows == 2) {
       if (who & 2) compute_row(std::integral_constant<int, 1>{}, ok);
@@ -643,24 +650,27 @@ __global__ __launch_bounds__(kWave* kSplit, 2) void sparse_attn_kernel(SaArgs a)
     for (int i = 0; i < kRows; ++i) {
       if (i >= rows) break;
       const float l_tot = sa_sum_x32(sa_sum_x16(l_run[i]));
-      const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+      const float inv = l_tot > 0.f ? 1.f / l_tot : ((seen >> i) & 1) ? NAN : 0.f;
 #pragma unroll
       for (int dt = 0; dt < 8; ++dt)
         sa_store4<OutT>(orow + i * static_cast<int64_t>(a.Hkv) * kSaG * kSaD + 16 * dt, o[i][dt] * inv);
     }
   } else {
     const float l_tot = sa_sum_x32(sa_sum_x16(l_run[0]));
-    // Each wave leaves (max, sum) per head and its O^T in its slot; then wave
-    // w combines dim tiles w, w + kSplit, ... of all of them.
+    // Each wave leaves (max, sum) per head and its O^T in its slot -- a max of
+    // -inf when it attended nothing; then wave w combines dim tiles w,
+    // w + kSplit, ... of all of them.
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt) *reinterpret_cast<f32x4*>(slot + 1024 * dt + 16 * lane) = o[0][dt];
-    if (g == 0) *reinterpret_cast<float2*>(slot + 8192 + 8 * s) = make_float2(m_run[0], l_tot);
+    if (g == 0) *reinterpret_cast<float2*>(slot + 8192 + 8 * s) = make_float2(seen != 0 ? m_run[0] : -INFINITY, l_tot);
     __syncthreads();
     float m[kSplit], l = 0.f, top = -3.402823466e38f;
+    bool any = false;
 #pragma unroll
     for (int w = 0; w < kSplit; ++w) {
       const float2 ml = *reinterpret_cast<const float2*>(lds + w * kSaWaveLds + 8192 + 8 * s);
       m[w] = ml.x;
+      any |= ml.x != -INFINITY;
       top = fmaxf(top, ml.x);
     }
 #pragma unroll
@@ -668,7 +678,7 @@ __global__ __launch_bounds__(kWave* kSplit, 2) void sparse_attn_kernel(SaArgs a)
       m[w] = __builtin_amdgcn_exp2f(m[w] - top);
       l += m[w] * (*reinterpret_cast<const float2*>(lds + w * kSaWaveLds + 8192 + 8 * s)).y;
     }
-    const float inv = l > 0.f ? 1.f / l : 0.f;
+    const float inv = l > 0.f ? 1.f / l : any ? NAN : 0.f;
     for (int dt = wave; dt < 8; dt += kSplit) {
       f32x4 v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
