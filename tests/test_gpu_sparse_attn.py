@@ -389,3 +389,21 @@ def test_infinite_scores(T, Hkv, B, slots, dev):
                          pd["token_pos_in_bs"], pd["seqlen_q"], head_group=Hkv) if slots else None
     got = sparse_paged_attention(**pd, slots=st, out_dtype=torch.float32).cpu()
     torch.testing.assert_close(got, exp, atol=ATOL, rtol=RTOL, equal_nan=True)
+
+
+@pytest.mark.parametrize("T,Hkv,B,slots", [(9, 2, 3, False), (9, 2, 3, True), (600, 2, 2, False),
+                                           (600, 2, 2, True), (1030, 4, 3, False)])
+def test_wrapped_block_ids(T, Hkv, B, slots, dev):
+    # Ids whose position id * 64 wraps int32: plus or minus 2^26 is the same
+    # block, plus 2^25 a negative position (nothing attended).
+    p = _problem(1300 + T, T=T, Hkv=Hkv, K=6, B=B, n_blocks=30, L=64 * 20, neg=0.1)
+    g = torch.Generator().manual_seed(T)
+    add = torch.tensor([0, 1 << 26, -(1 << 26), 1 << 25, 31 << 26, -(32 << 26)], dtype=torch.int64)
+    pick = torch.randint(0, 6, p["topk_idx"].shape, generator=g)
+    p["topk_idx"] = torch.where(p["topk_idx"] >= 0, p["topk_idx"] + add[pick], -1).to(torch.int32)
+    exp = oracle_attn(**p)
+    pd = {k: (v.to(dev) if isinstance(v, torch.Tensor) else v) for k, v in p.items()}
+    st = get_block_table(pd["topk_idx"], pd["block_table"], pd["token_to_bs"],
+                         pd["token_pos_in_bs"], pd["seqlen_q"], head_group=Hkv) if slots else None
+    got = sparse_paged_attention(**pd, slots=st, out_dtype=torch.float32).cpu()
+    torch.testing.assert_close(got, exp, atol=ATOL, rtol=RTOL)

@@ -325,6 +325,12 @@ struct SaBlock {
   uint32_t rows;
 };
 
+// Position of entry o of a block, wrapping int32 as the block table's (an id
+// past 2^25 can wrap to a live position: the product is unsigned).
+__device__ __forceinline__ int32_t sa_pos(int32_t id, int o) {
+  return static_cast<int32_t>(static_cast<uint32_t>(id) * 64u + static_cast<uint32_t>(o));
+}
+
 // The load of a block's table entries into `slot`, lane l's own key's entry
 // to word l: the slot table's, or block_table[b, min(p, L-1)]; zeros past the
 // last block.  One vector-memory operation, always issued.
@@ -338,7 +344,7 @@ __device__ __forceinline__ void sa_table(const SaArgs& a, const SaBlock& blk, ui
   } else if constexpr (kTable) {
     p = blk.run + kk;
   } else {
-    const int32_t pos = blk.id * 64 + kk;  // the block is live: no wrap
+    const int32_t pos = sa_pos(blk.id, kk);  // the block is live: >= 0
     p = blk.run + (pos < a.L - 1 ? pos : a.L - 1);
   }
   int saved;
@@ -352,7 +358,7 @@ __device__ __forceinline__ void sa_table(const SaArgs& a, const SaBlock& blk, ui
 template <bool kTable, bool kWide>
 __device__ __forceinline__ SaRowAt<kWide> sa_rows(const SaArgs& a, const SaBlock& blk, int h, int32_t tv) {
   const int lane = threadIdx.x & (kWave - 1);
-  const int32_t pos = blk.id * 64 + 4 * (lane & 15) + (lane >> 4);
+  const int32_t pos = sa_pos(blk.id, 4 * (lane & 15) + (lane >> 4));
   const uint32_t r = kTable ? static_cast<uint32_t>(tv)
                             : static_cast<uint32_t>(a.Hkv) * static_cast<uint32_t>(tv) + static_cast<uint32_t>(h);
   const bool ok = pos < blk.lim && r < static_cast<uint32_t>(a.n_rows);  // n_rows < 2^31: r >= 0 too
@@ -452,7 +458,7 @@ __global__ __launch_bounds__(kWave* kSplit, 2) void sparse_attn_kernel(SaArgs a)
   uint64_t live[kRows];
 #pragma unroll
   for (int i = 0; i < kRows; ++i) {
-    const int32_t p0 = static_cast<int32_t>(static_cast<uint32_t>(sel[i].lane_id) * 64u);
+    const int32_t p0 = sa_pos(sel[i].lane_id, 0);
     live[i] = __ballot(p0 >= 0 && p0 < sel[i].lim);
   }
   if constexpr (kSplit > 1) {
@@ -479,7 +485,7 @@ __global__ __launch_bounds__(kWave* kSplit, 2) void sparse_attn_kernel(SaArgs a)
       const int32_t id1 = __builtin_amdgcn_readlane(sel[1].lane_id, k1);
       const bool first = live[0] != 0 && (live[1] == 0 || !same || id0 <= id1);
       const int32_t least = sel[0].lim < sel[1].lim ? sel[0].lim : sel[1].lim;
-      const bool both = first && live[1] != 0 && same && id0 == id1 && id0 * 64 + 63 < least;
+      const bool both = first && live[1] != 0 && same && id0 == id1 && sa_pos(id0, 63) < least;
       if (first) live[0] &= live[0] - 1;
       if (!first || both) live[1] &= live[1] - 1;
       return first ? at_block(sel[0], k0, both ? 3 : 1) : at_block(sel[1], k1, 2);
