@@ -126,3 +126,20 @@ def test_other_groups_strided_inputs(Hq, Hkv, D, dev):
         if off == 8:
             assert torch.equal(out, base)
         torch.testing.assert_close(out.cpu(), exp, atol=1e-6, rtol=2e-5)
+
+
+def test_grid_of_2_to_24_pieces(dev):
+    # 65535 kv heads x (1 token piece + 256 sequences): more four-wave
+    # workgroups than a launch takes, so the scalar kernel runs.
+    Hkv, G, D, B, T, lk = 65535, 32, 8, 256, 2, 20
+    g = torch.Generator(device=dev).manual_seed(3)
+    q = torch.randn(T, Hkv * G, D, generator=g, device=dev).to(torch.bfloat16)
+    k = torch.randn(lk, Hkv, D, generator=g, device=dev).to(torch.bfloat16)
+    cu_q = torch.full((B + 1,), T, dtype=torch.int32, device=dev)
+    cu_k = torch.full((B + 1,), lk, dtype=torch.int32, device=dev)
+    cu_q[0] = cu_k[0] = 0
+    out = infllmv2_attn_stage1(q, k, None, cu_q, cu_k, max_seqlen_k=lk, causal=False)
+    x = (q.float().view(T, Hkv, G, 1, D) * k.float().permute(1, 0, 2).reshape(1, Hkv, 1, lk, D)).sum(-1)
+    exp = torch.softmax(x * D ** -0.5, -1).sum(2).transpose(0, 1)
+    torch.testing.assert_close(out[:, :, :lk], exp, atol=1e-6, rtol=2e-5)
+    assert not out[:, :, lk:].any()
