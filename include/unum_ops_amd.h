@@ -308,8 +308,9 @@ int unum_get_block_table(const int32_t* topk_idx, int64_t topk_stride_h,
  *   out[t, h*G+i] = sum_j softmax_j(scale * q[t,h*G+i] . K[row_j]) V[row_j]
  * over the attended entries (repeats counted), fp32 math, and 0 when (t, h)
  * has none.  Any finite scale is accepted (zero gives the mean of the
- * attended V rows, a negative one the softmax of the negated products).  G = Hq / Hkv must be 16 and D 128; K <= 64; q, the caches and
- * out 16-byte aligned.
+ * attended V rows, a negative one the softmax of the negated products).
+ * G = Hq / Hkv must be 16 and D 128; K <= 64; q, the caches and out 16-byte
+ * aligned; T * Hkv below 2^31.
  */
 int unum_sparse_paged_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h,
                                 const void* key_cache, const void* value_cache,

@@ -407,3 +407,28 @@ def test_wrapped_block_ids(T, Hkv, B, slots, dev):
                          pd["token_pos_in_bs"], pd["seqlen_q"], head_group=Hkv) if slots else None
     got = sparse_paged_attention(**pd, slots=st, out_dtype=torch.float32).cpu()
     torch.testing.assert_close(got, exp, atol=ATOL, rtol=RTOL)
+
+
+def test_more_than_2_to_24_shared_rows(dev):
+    # 2^24 + 16 (token, kv head) rows shared by four waves each: more than 2^32
+    # threads.  One sequence a token, all with one table row; one query, one
+    # block id and one limit for all, so every row's output is the first's.
+    Hkv, T = 16, (1 << 20) + 1
+    if torch.cuda.mem_get_info(dev)[0] < 80 << 30:
+        pytest.skip("needs 80 GiB of GPU memory")
+    g = torch.Generator().manual_seed(5)
+    q1 = torch.randn(1, 16 * Hkv, 128, generator=g).to(torch.bfloat16)
+    kc, vc = (torch.randn(2, 64, Hkv, 128, generator=g).to(torch.bfloat16) for _ in range(2))
+    tab = torch.arange(128, dtype=torch.int32)[None]
+    idx = torch.ones(Hkv, 1, 1, dtype=torch.int32)
+    one = torch.tensor([100], dtype=torch.int32)
+    exp = oracle_attn(q1, kc, vc, 16 * Hkv, Hkv, 128 ** -0.5, idx, tab,
+                      torch.zeros(1, dtype=torch.int32), one, one)
+    out = sparse_paged_attention(
+        q1.to(dev).expand(T, -1, -1), kc.to(dev), vc.to(dev), 16 * Hkv, Hkv, 128 ** -0.5,
+        idx.to(dev).expand(-1, T, -1), tab.to(dev).expand(T, -1),
+        torch.arange(T, dtype=torch.int32, device=dev), one.to(dev), one.to(dev))
+    torch.testing.assert_close(out[:1].float().cpu(), exp, atol=ATOL, rtol=RTOL_BF16_OUT)
+    bits = out.view(torch.int16)
+    for a in range(0, T, 1 << 16):
+        assert bool((bits[a:a + (1 << 16)] == bits[:1]).all()), a

@@ -385,10 +385,12 @@ __device__ __forceinline__ void sa_wait() {
 // workgroups of a head go to one XCD, so that the rows that neighbouring tokens
 // both attend (those of one sequence, to begin with) are fetched into one L2,
 // and groups are dealt in turn, so that the XCDs get equal work also where
-// contexts grow along t.
+// contexts grow along t.  The grid is rows of 2^kSaGridShift workgroups: one
+// dimension holds less than 2^32 threads, 2^24 four-wave workgroups.
+constexpr int kSaGridShift = 20;
 template <int kRows>
 __device__ __forceinline__ bool sa_row(const SaArgs& a, int& t, int& h) {
-  const uint32_t id = blockIdx.x;
+  const uint32_t id = (blockIdx.y << kSaGridShift) + blockIdx.x;
   const uint32_t j = id >> 3;
   const uint32_t group = ((j >> a.gshift) << 3) + (id & 7);
   const uint32_t units = (static_cast<uint32_t>(a.T) + kRows - 1) / kRows;
@@ -924,7 +926,12 @@ extern "C" int unum_sparse_paged_attention(
   a.gshift = 0;
   while (a.gshift < 4 && ((units * Hkv) >> a.gshift) >= 128) ++a.gshift;
   const int64_t groups = ((units + (int64_t{1} << a.gshift) - 1) >> a.gshift) * Hkv;
-  const dim3 grid(static_cast<unsigned>(((groups + 7) / 8) << (a.gshift + 3)));
+  const int64_t wgs = ((groups + 7) / 8) << (a.gshift + 3);
+  UNUM_REQUIRE(wgs <= INT32_MAX, "%s: size exceeds the kernel's index range (%lld tokens x %lld kv heads)",
+               op, (long long)T, (long long)Hkv);
+  constexpr int64_t kGridRow = int64_t{1} << kSaGridShift;
+  const dim3 grid(static_cast<unsigned>(wgs < kGridRow ? wgs : kGridRow),
+                  static_cast<unsigned>((wgs + kGridRow - 1) / kGridRow));
   hipStream_t s = static_cast<hipStream_t>(stream);
   auto launch = [&](auto o, auto tab, auto w) {
     using OutT = decltype(o);
