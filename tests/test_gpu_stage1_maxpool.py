@@ -165,3 +165,32 @@ def test_decode_rows_pooled(q_lens, k_lens, causal, local, init, dev):
     exp_p = oracle_pool(scores.cpu(), d["cu_seqlens_q"], d["cu_seqlens_k"], cache,
                         16 * scores.shape[-1], mcl, local, init, oob="absent")
     np.testing.assert_array_equal(pooled.cpu().numpy(), exp_p)
+
+
+@pytest.mark.parametrize("q_lens,splits", [
+    ([1] * 64, False), ([300] + [0] * 255, False), ([1] * 400, False), ([500] + [0] * 511, True),
+    ([4] * 64, True),
+])
+def test_decode_kernel_or_key_splits(q_lens, splits, dev):
+    # The decode kernel reads a row's keys for every row: a batch padded with
+    # empty sequences that holds one long chunk runs the key splits, which write
+    # their workspace; the decode kernel leaves it alone.
+    from unum_ops_amd import _lib
+    B, T, keys = len(q_lens), sum(q_lens), 600
+    g = torch.Generator().manual_seed(T)
+    q = torch.randn(T, 32, 128, generator=g).to(torch.bfloat16).to(dev)
+    k = torch.randn(B * keys, 2, 128, generator=g).to(torch.bfloat16).to(dev)
+    cu_q = torch.tensor(np.concatenate([[0], np.cumsum(q_lens)]), dtype=torch.int32, device=dev)
+    cu_k = torch.arange(B + 1, dtype=torch.int32, device=dev) * keys
+    lib = _lib.load()
+    need = lib.unum_infllmv2_attn_stage1_workspace_size(B, T, 32, 2, 128, keys)
+    assert need > 0
+    ws = torch.full((need,), 0xA5, dtype=torch.uint8, device=dev)
+    nb = -(-(16 * keys + 16) // 64)
+    pooled = torch.empty(2, T, nb, device=dev)
+    st = lib.unum_infllmv2_attn_stage1_maxpool(
+        _lib.ptr(q), q.stride(0), q.stride(1), _lib.ptr(k), k.stride(0), k.stride(1),
+        _lib.ptr(cu_q), _lib.ptr(cu_k), None, _lib.ptr(pooled), B, T, B * keys, 32, 2, 128, keys,
+        640, 128 ** -0.5, 1, nb, 1, 1, _lib.ptr(ws), need, _lib.stream_ptr(q.device))
+    _lib.check(st, "infllmv2_attn_stage1_maxpool")
+    assert bool((ws != 0xA5).any()) == splits
