@@ -292,7 +292,11 @@ int unum_get_block_table(const int32_t* topk_idx, int64_t topk_stride_h,
  *                s*Hkv + h holds token slot s, kv head h
  *   topk_idx     int32 [Hkv, T, K] block ids, element strides (h, t, k)
  *   block_table  int32 [B, L] token-granular table, row stride bt_stride_b
- *                (unused when `slots` is given)
+ *                (unused when `slots` is given).  B also tells the launch how
+ *                many sequences the T tokens are of: a table with many more
+ *                rows than the batch has sequences gives the same result, but
+ *                a long chunk then runs as a batch of short ones would (4096
+ *                tokens: 1217 us with 256 rows, 683 with one)
  *   slots        optional int32 [T, Hkv, K*64] contiguous: get_block_table's
  *                output for these inputs with head_group = Hkv (NULL: the
  *                slots are computed from block_table)

@@ -432,3 +432,19 @@ def test_more_than_2_to_24_shared_rows(dev):
     bits = out.view(torch.int16)
     for a in range(0, T, 1 << 16):
         assert bool((bits[a:a + (1 << 16)] == bits[:1]).all()), a
+
+
+def test_one_token_a_sequence_takes_whole_rows(dev):
+    # 512 sequences of one token (1024 rows) and the same tokens 64 times over
+    # (64 tokens a sequence): both one row a wave or, in the larger, two, so the
+    # same bits.  (Rows shared by four waves sum in another order.)
+    p = _problem(1400, T=512, B=512, K=9, n_blocks=64, L=64 * 30)
+    p["token_to_bs"] = torch.randperm(512, generator=torch.Generator().manual_seed(1)).to(torch.int32)
+    pd = {k: (v.to(dev) if isinstance(v, torch.Tensor) else v) for k, v in p.items()}
+    once = sparse_paged_attention(**pd, out_dtype=torch.float32)
+    torch.testing.assert_close(once.cpu(), oracle_attn(**p), atol=ATOL, rtol=RTOL)
+    for name in ("query", "token_to_bs", "token_pos_in_bs"):
+        pd[name] = pd[name].repeat(64, *[1] * (pd[name].dim() - 1))
+    pd["topk_idx"] = pd["topk_idx"].repeat(1, 64, 1)
+    many = sparse_paged_attention(**pd, out_dtype=torch.float32)
+    assert torch.equal(many, once.repeat(64, 1, 1))

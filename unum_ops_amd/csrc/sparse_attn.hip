@@ -914,14 +914,19 @@ extern "C" int unum_sparse_paged_attention(
   // that are alike; else four waves share a row.  Measured, whole / shared:
   // 64 sequences x 1 token 96 / 49 us, x 8 tokens 231 / 202, x 16 tokens
   // 420 / 318 (fewer rows at once keep a sequence's blocks in the L2); one
-  // sequence x 512 tokens 105 / 103, x 1024 193 / 205, x 2048 363 / 403.
-  const bool whole = rows >= 1024 && T >= 64 * B;
+  // sequence x 512 tokens 105 / 103, x 1024 193 / 205, x 2048 363 / 403.  At
+  // most one token a sequence, no row meets another's blocks in the L2 and
+  // sharing a row only costs its combination: 512 sequences x 2 blocks
+  // 15.6 / 18.2, x 64 blocks 358 / 366; 2048 x 2 blocks 50.6 / 59.9.  (B, the
+  // table's rows, stands for the sequences of the batch: they are counted on
+  // the device only.)
+  const bool whole = rows >= 1024 && (T >= 64 * B || T <= B);
   // Two rows a wave where that still fills the chip (eight waves a CU).
   // Measured, one row a wave / two, neighbours' selections 6, 24 and 67 %
   // alike: 4096 tokens of 2 heads 1738 / 1564, 925 / 722 and 664 / 564 us,
   // 2048 tokens 687 / 573, 373 / 344 and 344 / 284, 1024 tokens (a wave a
   // SIMD) 322 / 299, 192 / 208 and 173 / 184.
-  const bool pairs = whole && !slots && rows >= 4096;
+  const bool pairs = whole && T > B && !slots && rows >= 4096;
   const int64_t units = pairs ? (T + 1) / 2 : T;  // workgroups of a head
   a.gshift = 0;
   while (a.gshift < 4 && ((units * Hkv) >> a.gshift) >= 128) ++a.gshift;
