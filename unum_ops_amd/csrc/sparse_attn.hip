@@ -213,11 +213,27 @@ __device__ __forceinline__ void sa_store4<uint16_t>(uint16_t* p, f32x4 v) {
   *reinterpret_cast<uint2*>(p) = make_uint2(lo, hi);
 }
 
-// 16-byte chunk c of a row in LDS lies at chunk c ^ sa_swz(key): distinct
-// for the 16 keys of a tile, and even for its first eight, odd for the
-// others, so the aligned chunk pairs that the transposing reads of V take
-// from eight keys are distinct too.
-__device__ __forceinline__ int sa_swz(int key) { return ((key & 7) << 1) | ((key >> 3) & 1); }
+// 16-byte chunk c of a row in LDS lies at chunk c ^ sa_swz(key).  A K operand
+// read takes chunk c of keys 0-3 and 12-15 and chunk c ^ 1 of keys 4-11 in one
+// service (lds_b128_free), so the values of either eight keys are four pairs
+// {2i, 2i + 1}; those of keys 0-7, and of 8-15, lie in different pairs, so the
+// aligned chunk pairs that the transposing reads of V take from eight keys are
+// distinct too.  (Keys 0-7 even, 8-15 odd, in order, met twice on every K
+// read: a third of the LDS's active cycles.)
+__host__ __device__ constexpr int sa_swz(int key) {
+  return (((key & 7) ^ (4 * ((key >> 3) & 1))) << 1) | ((key >> 3) & 1);
+}
+constexpr bool sa_lds_free() {
+  struct K { constexpr int operator()(int lane) const { return 16 * (lane & 15) + ((lane >> 4) ^ sa_swz(lane & 15)); } };
+  if (!lds_b128_free(K{})) return false;
+  for (int g = 0; g < 4; g += 2) {  // V: 32 lanes, eight keys, a chunk pair of each
+    uint32_t pairs = 0;
+    for (int key = 4 * g; key < 4 * g + 8; ++key) pairs |= 1u << (sa_swz(key) >> 1);
+    if (pairs != 0xFFu) return false;
+  }
+  return true;
+}
+static_assert(sa_lds_free(), "K and V operand reads meet no LDS bank twice");
 
 typedef __attribute__((address_space(3))) void* sa_lds_void;
 __device__ __forceinline__ uint32_t sa_lds_at(const void* p) {
