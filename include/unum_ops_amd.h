@@ -161,12 +161,18 @@ int unum_infllmv2_attn_stage1_noalloc(const void* q, int64_t q_stride_t, int64_t
  *   workspace / workspace_bytes  as unum_infllmv2_attn_stage1 (size from
  *          unum_infllmv2_attn_stage1_workspace_size): with it, rows over 512
  *          keys run the key-split kernels, pooling in their second pass;
- *          NULL runs whole rows.  Rows of at most 512 keys need none.
+ *          NULL runs whole rows.  Rows of at most 512 keys need none, and
+ *          decode batches leave it unused: at most two new tokens per
+ *          sequence, rows of at most 4096 keys, and either as many tokens as
+ *          sequences or at most 3 rows (token, kv head) per CU.
  * Other arguments as unum_infllmv2_attn_stage1 and unum_max_pooling_1d_varlen.
  * Fused on the MFMA paths (G = 16, D = 128, 16-byte aligned q/k, scale > 0):
- * rows of at most 512 keys pool in the LDS-resident kernel, longer rows in
- * the key-streaming kernels.  Other shapes return UNUM_ERR_UNSUPPORTED; run
- * unum_infllmv2_attn_stage1 and unum_max_pooling_1d_varlen there.
+ * rows of at most 512 keys pool in the LDS-resident kernel, decode batches in
+ * a kernel of one workgroup a row, other rows in the key-streaming kernels.
+ * Other shapes return UNUM_ERR_UNSUPPORTED; run unum_infllmv2_attn_stage1 and
+ * unum_max_pooling_1d_varlen there.  On decode batches unum_infllmv2_attn_stage1
+ * keeps f16 exponentials, this entry f16 probabilities: their scores differ in
+ * the last f16 bits.
  */
 int unum_infllmv2_attn_stage1_maxpool(const void* q, int64_t q_stride_t, int64_t q_stride_h,
                                       const void* k, int64_t k_stride_t, int64_t k_stride_h,
@@ -311,7 +317,9 @@ int unum_get_block_table(const int32_t* topk_idx, int64_t topk_stride_h,
  * (wrapping int32) -- lies in [0, n_rows).  Then
  *   out[t, h*G+i] = sum_j softmax_j(scale * q[t,h*G+i] . K[row_j]) V[row_j]
  * over the attended entries (repeats counted), fp32 math, and 0 when (t, h)
- * has none.  Any finite scale is accepted (zero gives the mean of the
+ * has none.  A score of -inf has weight 0; where every attended score of a
+ * head is -inf there is no softmax and its output is NaN, as where one is +inf
+ * or NaN.  Any finite scale is accepted (zero gives the mean of the
  * attended V rows, a negative one the softmax of the negated products).
  * G = Hq / Hkv must be 16 and D 128; K <= 64; q, the caches and out 16-byte
  * aligned; T * Hkv below 2^31.

@@ -448,3 +448,25 @@ def test_one_token_a_sequence_takes_whole_rows(dev):
     pd["topk_idx"] = pd["topk_idx"].repeat(1, 64, 1)
     many = sparse_paged_attention(**pd, out_dtype=torch.float32)
     assert torch.equal(many, once.repeat(64, 1, 1))
+
+
+@pytest.mark.parametrize("T,slots", [(9, False), (9, True), (1100, False), (1100, True), (4100, False)])
+def test_wide_caches_every_instance(T, slots, dev):
+    # Whole addresses (caches past 4 GiB) with rows shared by four waves, one
+    # row a wave and two rows a wave, and the first two from a slot table: the
+    # bits of the same rows in caches below 4 GiB, where the other tests check
+    # every instance against the oracle.
+    p = _problem(1500 + T, T=T, Hkv=1, K=6, n_blocks=1024, L=640)
+    p["block_table"] = torch.randint(65536 - 640, 65536 + 40, p["block_table"].shape,
+                                     dtype=torch.int32, generator=torch.Generator().manual_seed(T))
+    pd = {k: (v.to(dev) if isinstance(v, torch.Tensor) else v) for k, v in p.items()}
+    st = get_block_table(pd["topk_idx"], pd["block_table"], pd["token_to_bs"],
+                         pd["token_pos_in_bs"], pd["seqlen_q"], head_group=1) if slots else None
+    near = sparse_paged_attention(**pd, slots=st, out_dtype=torch.float32)
+    assert not torch.isnan(near).any() and near.any()
+    row = 32776
+    for name in ("key_cache", "value_cache"):
+        big = torch.empty(65536 * row, dtype=torch.bfloat16, device=dev)
+        pd[name] = big.as_strided((1024, 64, 1, 128), (64 * row, row, row, 1))
+        pd[name].copy_(p[name])
+    assert torch.equal(sparse_paged_attention(**pd, slots=st, out_dtype=torch.float32), near)

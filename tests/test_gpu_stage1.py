@@ -83,8 +83,9 @@ def test_peaky_keys(peaky, dev):
 
 
 def test_generic_kernel_shapes(dev):
-    # G = 8 and D = 64 run the general kernel
-    for Hq, Hkv, D in [(32, 4, 128), (16, 1, 64), (32, 2, 64)]:
+    # G = 8 and D = 64 run the group kernel, G = 33, D = 100 and D = 264 the
+    # scalar one
+    for Hq, Hkv, D in [(32, 4, 128), (16, 1, 64), (32, 2, 64), (66, 2, 64), (32, 2, 100), (4, 2, 264)]:
         d = workloads.stage1_inputs([20, 33], [400, 700], Hq=Hq, Hkv=Hkv, D=D, seed=Hq + D)
         _check(d, _run(d, dev))
 

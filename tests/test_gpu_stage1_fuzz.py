@@ -86,11 +86,13 @@ def test_random_batches(seed, dev):
     np.testing.assert_array_equal(pooled.cpu().numpy(), exp_p)
 
 
-@pytest.mark.parametrize("seed", range(8))
+@pytest.mark.parametrize("seed", range(12))
 def test_random_generic_shapes(seed, dev):
-    # head groups other than 16 and head dims other than 128: the generic kernel
+    # head groups other than 16 and head dims other than 128: the group kernel,
+    # and from seed 8 the scalar one
     q_lens, ctx, _, _, causal = _batch(4 * seed)  # rows of at most 512 keys
-    hq, hkv, D = [(32, 4, 128), (16, 1, 64), (8, 8, 128), (24, 2, 64)][seed % 4]
+    hq, hkv, D = ([(32, 4, 128), (16, 1, 64), (8, 8, 128), (24, 2, 64)] if seed < 8 else
+                  [(34, 1, 64), (16, 2, 92), (66, 2, 128), (6, 2, 260)])[seed % 4]
     d = workloads.stage1_inputs(q_lens, ctx, Hq=hq, Hkv=hkv, D=D, seed=seed, raw_keys=False)
     print(f"seed {seed}: q {q_lens} ctx {ctx} Hq {hq} Hkv {hkv} D {D} causal {causal}", flush=True)
     msk = max(d["max_seqlen_k"], 1)

@@ -14,8 +14,8 @@
 Each case runs every kernel family: the LDS-resident kernel (at most 512
 columns), the key-streaming kernels (whole rows and key splits), the decode
 kernel (at most two new tokens per sequence), the row-MFMA kernel (a
-non-positive scale) and the generic kernel (four heads per group, or a q
-whose base is not 16-byte aligned).
+non-positive scale), the group kernel (four heads per group) and the generic
+kernel (33 heads per group, or a q whose base is not 16-byte aligned).
 """
 
 import ctypes
@@ -43,7 +43,8 @@ CASES = {
     "stream_whole": ([64, 64], [3000, 900], 1000, False, 32, SCALE, 0),  # no workspace
     "decode": ([1, 2, 1], [3000, 2500, 800], 1000, False, 32, SCALE, 0),  # Tq <= 2B
     "row_mfma": ([40, 300], [700, 200], 300, False, 32, -SCALE, 0),      # non-positive scale
-    "generic_g4": ([40, 70], [700, 200], 300, False, 8, SCALE, 0),       # 4 heads per group
+    "group_g4": ([40, 70], [700, 200], 300, False, 8, SCALE, 0),         # 4 heads per group
+    "generic_g33": ([40, 70], [700, 200], 300, False, 66, SCALE, 0),     # 33 heads per group
     "generic_unaligned": ([40, 70], [700, 200], 300, False, 32, SCALE, 1),  # q base + 2 bytes
 }
 
@@ -147,7 +148,7 @@ def test_negative_first_key_offset_reads_nothing(case, dev):
     torch.testing.assert_close(out[:, q_lens[0]:], exp[:, q_lens[0]:], atol=ATOL, rtol=RTOL)
 
 
-@pytest.mark.parametrize("case", ["lds", "stream_split", "decode", "row_mfma", "generic_g4"])
+@pytest.mark.parametrize("case", ["lds", "stream_split", "decode", "row_mfma", "group_g4", "generic_g33"])
 def test_keys_past_the_end_of_k_read_as_zero(case, dev):
     # The last sequence claims more keys than k holds: its keys at rows past
     # the end of k score as zero keys, on every path alike.  The oracle gets

@@ -1,6 +1,6 @@
 """GPU parity of the fused stage-1 + max-pool entry point (fused in the
-LDS-resident kernel for rows of at most 512 keys, in the K-streaming kernels
-for longer rows).
+LDS-resident kernel for rows of at most 512 keys, in the decode kernel or the
+K-streaming kernels for longer rows).
 
 The pooled scores must equal, bit for bit, the max-pool the oracle computes
 from the scores the same kernel wrote (``return_scores``), and the scores must
@@ -13,10 +13,12 @@ import pytest
 import torch
 
 from oracle.maxpool import max_pooling_1d_varlen as oracle_pool
-from oracle.stage1 import infllmv2_attn_stage1 as oracle_stage1
+from oracle.stage1 import infllmv2_attn_stage1 as oracle_stage1, visible_counts
 import workloads
 from unum_ops_amd import _lib
-from unum_ops_amd.infllm_v2 import infllmv2_attn_stage1_maxpool
+from unum_ops_amd.infllm_v2 import (infllmv2_attn_stage1, infllmv2_attn_stage1_maxpool,
+                                    max_pooling_1d_varlen)
+from unum_ops_amd.pipeline import topk_blocks
 
 pytestmark = pytest.mark.gpu
 
@@ -167,6 +169,63 @@ def test_decode_rows_pooled(q_lens, k_lens, causal, local, init, dev):
     np.testing.assert_array_equal(pooled.cpu().numpy(), exp_p)
 
 
+@pytest.mark.parametrize("causal", [True, False])
+def test_decode_rows_orphans_and_offsets(causal, dev):
+    # The decode kernel with tokens before the first sequence and after the
+    # last, and a first sequence whose keys lie before k (they read as zero
+    # keys: every visible score is 16 / vis).
+    k_lens = [700, 600, 900, 3000, 1500, 1400]
+    d = workloads.stage1_inputs([1, 2, 1, 0, 1, 1], [16 * (n - 1) + 32 for n in k_lens], seed=40,
+                                raw_keys=False)
+    d["q"] = torch.cat([d["q"], d["q"]])[:11]            # 2 + 6 + 3 tokens, at most 2 a sequence
+    d["cu_seqlens_q"] = d["cu_seqlens_q"] + 2
+    d["cu_seqlens_k"] = d["cu_seqlens_k"].clone()
+    d["cu_seqlens_k"][0] = -5
+    ctx = 16 * 1500
+    args = [d[n].to(dev) for n in ("q", "k", "cu_seqlens_q", "cu_seqlens_k")]
+    kw = dict(max_seqlen_k=1500, causal=causal)
+    pooled, scores = infllmv2_attn_stage1_maxpool(*args, ctx, return_scores=True, **kw)
+    assert torch.equal(infllmv2_attn_stage1_maxpool(*args, ctx, **kw), pooled)
+    exp = oracle_stage1(d["q"], d["k"], None, d["cu_seqlens_q"], d["cu_seqlens_k"].clamp(min=0),
+                        max_seqlen_k=1500, causal=causal)
+    vis = 705 if not causal else int(visible_counts(np.arange(1), 1, 705)[0])
+    exp[:, 2] = 0.0
+    exp[:, 2, :vis] = 16.0 / vis
+    scores = scores.cpu()
+    torch.testing.assert_close(scores, exp, atol=1e-3, rtol=1e-2)
+    assert not scores[:, :2].any() and not scores[:, 8:].any()
+    exp_p = oracle_pool(scores, d["cu_seqlens_q"], d["cu_seqlens_k"], torch.zeros(6, dtype=torch.int32),
+                        16 * scores.shape[-1], ctx, 1, 1, oob="absent")
+    np.testing.assert_array_equal(pooled.cpu().numpy(), exp_p)
+
+
+def test_decode_ids_against_the_two_ops(dev):
+    # Plain stage 1 keeps a decode row's probabilities as f16 exponentials times
+    # f16 weights, the fused entry rounds each probability to f16.  On nearly
+    # flat rows of up to 3800 keys, as here, all of them are normal f16 values
+    # (2^-10 truncated, 2^-11 for a weight; below 2^-14 a probability is off by
+    # 2^-24, 16 of them by 2^-20): the two are within 2^-8 of a score and 2^-20,
+    # and select the same blocks but for those that near to the K-th score.
+    d = workloads.stage1_inputs([1] * 64, [16384 + 700 * i for i in range(64)], seed=41, raw_keys=False)
+    args = [d[n].to(dev) for n in ("q", "k", "cu_seqlens_q", "cu_seqlens_k")]
+    ctx, K = 16384 + 700 * 63, 64
+    fused = infllmv2_attn_stage1_maxpool(*args, ctx, max_seqlen_k=d["max_seqlen_k"], causal=True)
+    sc = infllmv2_attn_stage1(args[0], args[1], None, *args[2:], max_seqlen_k=d["max_seqlen_k"], causal=True)
+    chain = max_pooling_1d_varlen(sc, *args[2:], torch.zeros(64, dtype=torch.int32, device=dev),
+                                  16 * sc.shape[-1], ctx, 1, 1)
+    fin = torch.isfinite(chain)
+    assert torch.equal(fin, torch.isfinite(fused)) and torch.equal(chain[~fin], fused[~fin])
+    far = (fused - chain).abs() - (2 ** -8 * chain + 2 ** -20)
+    assert float(far[fin].max()) <= 0
+    a, b = topk_blocks(fused, K).cpu(), topk_blocks(chain, K).cpu()
+    chain = chain.cpu()
+    for h in range(2):
+        for t in range(64):
+            kth = float(chain[h, t, b[h, t].long()].min())
+            for i in set(a[h, t].tolist()) ^ set(b[h, t].tolist()):
+                assert abs(float(chain[h, t, i]) - kth) <= 2 ** -7 * kth + 2 ** -19, (h, t, i)
+
+
 @pytest.mark.parametrize("q_lens,splits", [
     ([1] * 64, False), ([300] + [0] * 255, False), ([1] * 400, False), ([500] + [0] * 511, True),
     ([4] * 64, True),
@@ -175,7 +234,6 @@ def test_decode_kernel_or_key_splits(q_lens, splits, dev):
     # The decode kernel reads a row's keys for every row: a batch padded with
     # empty sequences that holds one long chunk runs the key splits, which write
     # their workspace; the decode kernel leaves it alone.
-    from unum_ops_amd import _lib
     B, T, keys = len(q_lens), sum(q_lens), 600
     g = torch.Generator().manual_seed(T)
     q = torch.randn(T, 32, 128, generator=g).to(torch.bfloat16).to(dev)

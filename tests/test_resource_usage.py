@@ -84,7 +84,8 @@ def test_other_kernels_use_no_scratch(name, all_usage):
 def test_every_kernel_instance_reported(usage):
     kinds = {k: sum(1 for n in usage if k in n) for k in
              ("stage1_lds_kernel", "stage1_stream_kernel", "stage1_decode_kernel",
-              "stage1_mfma_kernel", "stage1_generic_kernel")}
+              "stage1_decode_pool_kernel", "stage1_group_kernel", "stage1_mfma_kernel",
+              "stage1_generic_kernel")}
     assert all(v > 0 for v in kinds.values()), kinds
     assert all("ScratchSize" in v and "Occupancy" in v and "VGPRs" in v for v in usage.values())
     # The LDS-resident kernel's largest rows are known to need more than 128 VGPRs.

@@ -88,8 +88,8 @@ def infllmv2_attn_stage1(q, k, v, cu_seqlens_q, cu_seqlens_k, cu_seqlens_v=None,
         return out.zero_()
     lib = _lib.load()
     # Rows over 512 keys split their keys between workgroups through a
-    # small workspace (about 1 KiB per 16 rows and split); decode
-    # batches run one workgroup per row and need none.
+    # small workspace (about 1 KiB per 16 rows and split); decode batches
+    # run one workgroup per row and leave it unused.
     ws, ws_bytes = _lib.stage1_workspace(lib, dev, batch, total_q, n_heads, n_kv_heads, head_dim,
                                          max_seqlen_k)
     st = _lib.call(
@@ -165,10 +165,13 @@ def infllmv2_attn_stage1_maxpool(q, k, cu_seqlens_q, cu_seqlens_k, max_context_l
     init_blocks)`` -- each row pooled in place, as the selection pipeline
     chains the two ops -- computed in one kernel, so the fp32 scores only go
     to HBM when ``return_scores`` asks for them (then ``(pooled, scores)``):
-    rows of at most 512 keys pool in the LDS-resident stage-1 kernel, longer
-    rows in the key-streaming kernels.  Shapes off the MFMA paths (G != 16,
-    D != 128, ...) and ``block_size / stride`` other than 64 / 16 run the two
-    ops separately.
+    rows of at most 512 keys pool in the LDS-resident stage-1 kernel, decode
+    rows of at most 4096 keys in a kernel of one workgroup a row, other rows in
+    the key-streaming kernels.  Shapes off the MFMA paths (G != 16, D != 128,
+    ...) and ``block_size / stride`` other than 64 / 16 run the two ops
+    separately.  On decode batches ``infllmv2_attn_stage1`` alone rounds
+    otherwise (f16 exponentials, not f16 probabilities), so the two ops' scores
+    differ from these in the last f16 bits.
     """
     op = "infllmv2_attn_stage1_maxpool"
     dev = require_gpu(op, q, k, cu_seqlens_q, cu_seqlens_k)
@@ -218,7 +221,7 @@ def infllmv2_attn_stage1_maxpool(q, k, cu_seqlens_q, cu_seqlens_k, max_context_l
         return (pooled, scores) if return_scores else pooled
     lib = _lib.load()
     # The key-split workspace of stage 1: rows over 512 keys then pool in
-    # the split kernels' second pass.
+    # the split kernels' second pass (decode batches leave it unused).
     ws, ws_bytes = _lib.stage1_workspace(lib, dev, batch, total_q, n_heads, n_kv_heads, head_dim,
                                          max_seqlen_k)
     st = _lib.call(

@@ -141,14 +141,17 @@ def select_blocks(q, k, cu_seqlens_q, cu_seqlens_k, block_table, token_to_bs, to
     is the slot multiplier of ``get_block_table`` (default ``Hkv``, as the
     reference's exported Triton functions use).  With
     ``return_intermediates`` the scores, pooled scores and block ids are
-    returned too, as ``(table, scores, pooled, topk_idx)``.
+    returned too, as ``(table, scores, pooled, topk_idx)`` (on decode batches
+    from scores that differ from the fused ones by their rounding to f16, so a
+    near-tie for the last block may go the other way).
     """
     op = "select_blocks"
     dev = require_gpu(op, q, k, cu_seqlens_q, cu_seqlens_k, block_table)
     if not return_intermediates:
         # The scores are not wanted: stage 1 pools its rows in the kernel
         # (the score tensor never goes to HBM), then the top-k runs over the
-        # pooled rows -- the same ids as the chain below, bit for bit.
+        # pooled rows -- the ids of the chain below, bit for bit, but on decode
+        # batches (see infllmv2_attn_stage1_maxpool).
         pooled = infllmv2_attn_stage1_maxpool(q, k, cu_seqlens_q, cu_seqlens_k, max_context_len,
                                               max_seqlen_k=max_seqlen_k,
                                               softmax_scale=softmax_scale, causal=causal,
