@@ -95,7 +95,8 @@ def parse():
                                        "maxpool_cfg5", "maxpool_topk", "maxpool_topk_cfg5",
                                        "compress_keys_cfg5", "stage1_maxpool",
                                        "stage1_maxpool_cfg5", "stage1_cfg4", "stage1_decode",
-                                       "stage1_peaky", "stage1_cfg5_h16", "maxpool_cfg5_h16",
+                                       "stage1_maxpool_decode", "stage1_group8",
+                                       "stage2_decode", "stage1_peaky", "stage1_cfg5_h16", "maxpool_cfg5_h16",
                                        "block_table_cfg5_h16", "block_table_cfg4",
                                        "stage1_maxpool_cfg4", "stage2_cfg5", "stage2_cfg4",
                                        "topk_cfg5", "select_cfg5", "stage2_gather_cfg5",
@@ -115,7 +116,8 @@ def build_inputs(dev):
     import torch
 
     from tests import workloads
-    from unum_ops_amd.infllm_v2 import infllmv2_attn_stage1, max_pooling_1d_varlen
+    from unum_ops_amd.infllm_v2 import (infllmv2_attn_stage1, infllmv2_attn_stage1_maxpool,
+                                        max_pooling_1d_varlen)
     from unum_ops_amd.pipeline import topk_blocks
 
     t0 = time.time()
@@ -159,7 +161,19 @@ def build_inputs(dev):
     pd = workloads.pipeline_inputs([1] * 64, [32768] * 64, raw_keys=False)
     c5["decode"] = dict(q=pd["q"].to(dev), k=pd["k"].to(dev), cu_q=pd["cu_seqlens_q"].to(dev),
                         cu_k=pd["cu_seqlens_k"].to(dev), max_seqlen_k=pd["max_seqlen_k"],
-                        cu_q_cpu=pd["cu_seqlens_q"], cu_k_cpu=pd["cu_seqlens_k"])
+                        cu_q_cpu=pd["cu_seqlens_q"], cu_k_cpu=pd["cu_seqlens_k"],
+                        max_context_len=pd["max_context_len"],
+                        bt={n: pd[n].to(dev) for n in ("block_table", "token_to_bs",
+                                                       "token_pos_in_bs", "seqlen_q")})
+    cd = c5["decode"]
+    cd["bt"]["topk_idx"] = topk_blocks(
+        infllmv2_attn_stage1_maxpool(cd["q"], cd["k"], cd["cu_q"], cd["cu_k"],
+                                     cd["max_context_len"], max_seqlen_k=cd["max_seqlen_k"]), 64)
+    # Eight query heads a kv head: a prefill.
+    p8 = workloads.stage1_inputs([2000, 2400], [2000, 2400], Hq=32, Hkv=4, seed=8)
+    c5["group8"] = dict(q=p8["q"].to(dev), k=p8["k"].to(dev), cu_q=p8["cu_seqlens_q"].to(dev),
+                        cu_k=p8["cu_seqlens_k"].to(dev), max_seqlen_k=p8["max_seqlen_k"],
+                        cu_q_cpu=p8["cu_seqlens_q"], cu_k_cpu=p8["cu_seqlens_k"])
     # cfg5's Hq16/Hkv1 variant through the same stages (H = 1 everywhere).
     p6 = workloads.cfg5_pipeline(Hq=16, Hkv=1)
     q6, k6 = p6["q"].to(dev), p6["k"].to(dev)
@@ -308,6 +322,23 @@ def main():
         return infllmv2_attn_stage1(cd["q"], cd["k"], None, cd["cu_q"], cd["cu_k"],
                                     max_seqlen_k=cd["max_seqlen_k"], causal=True)
 
+    def op_stage1_maxpool_decode():
+        return infllmv2_attn_stage1_maxpool(cd["q"], cd["k"], cd["cu_q"], cd["cu_k"],
+                                            cd["max_context_len"],
+                                            max_seqlen_k=cd["max_seqlen_k"], causal=True)
+
+    def op_stage2_decode():
+        b = cd["bt"]
+        return sparse_paged_attention(cd["q"], c4["kv"][0], c4["kv"][1], 32, 2, 128 ** -0.5,
+                                      b["topk_idx"], b["block_table"], b["token_to_bs"],
+                                      b["token_pos_in_bs"], b["seqlen_q"])
+
+    c8 = c5["group8"]
+
+    def op_stage1_group8():
+        return infllmv2_attn_stage1(c8["q"], c8["k"], None, c8["cu_q"], c8["cu_k"],
+                                    max_seqlen_k=c8["max_seqlen_k"], causal=True)
+
     def op_compress_cfg5():
         return compress_keys(c5["raw"], c5["cu_raw"], plan=plan5)
 
@@ -407,6 +438,8 @@ def main():
              ("compress_keys_cfg5", op_compress_cfg5), ("stage1_maxpool", op_stage1_maxpool),
              ("stage1_maxpool_cfg5", op_stage1_maxpool_cfg5), ("stage1_cfg4", op_stage1_cfg4),
              ("stage1_decode", op_stage1_decode), ("stage1_peaky", op_stage1_peaky),
+             ("stage1_maxpool_decode", op_stage1_maxpool_decode),
+             ("stage1_group8", op_stage1_group8), ("stage2_decode", op_stage2_decode),
              ("stage1_cfg5_h16", op_stage1_cfg5_h16), ("maxpool_cfg5_h16", op_maxpool_cfg5_h16),
              ("block_table_cfg5_h16", op_block_table_cfg5_h16),
              ("block_table_cfg4", op_block_table_cfg4),
@@ -539,6 +572,27 @@ def main():
                                       config=f"decode: 64 sequences of 1 new token after 32768 "
                                              f"cached, Hq32/Hkv2/D128, fp32 out [2,64,{ncols}] "
                                              f"(not a BASELINE config)")
+    if "stage1_maxpool_decode" in per_op:
+        # the scores not written, the pooled blocks written
+        flop, nbytes, _ = workloads.stage1_work(cd["cu_q_cpu"], cd["cu_k_cpu"], 32, 2, 128, 0)
+        nblk = -(-cd["max_context_len"] // 64)
+        nbytes += 4 * 2 * 64 * nblk
+        t = per_op["stage1_maxpool_decode"] * 1e-3
+        comps["stage1_maxpool_decode"] = dict(
+            us=per_op["stage1_maxpool_decode"] * 1e3, tflops=flop / t / 1e12, gbs=nbytes / t / 1e9,
+            pct_hbm_peak=100 * nbytes / t / 1e9 / PEAK_HBM_GBS, flop=flop, bytes=nbytes, bound="hbm",
+            config=f"stage1_decode fused with the max-pool: pooled fp32 [2,64,{nblk}] only (scores "
+                   f"not stored)")
+    if "stage1_group8" in per_op:
+        ncols = -(-c8["max_seqlen_k"] // 128) * 128
+        flop, nbytes, _ = workloads.stage1_work(c8["cu_q_cpu"], c8["cu_k_cpu"], 32, 4, 128, ncols)
+        t = per_op["stage1_group8"] * 1e-3
+        comps["stage1_group8"] = dict(
+            us=per_op["stage1_group8"] * 1e3, tflops=flop / t / 1e12,
+            pct_bf16_mfma_peak=100 * flop / t / 1e12 / PEAK_BF16_TFLOPS, gbs=nbytes / t / 1e9,
+            pct_hbm_peak=100 * nbytes / t / 1e9 / PEAK_HBM_GBS, flop=flop, bytes=nbytes, bound="hbm",
+            config=f"prefill of 2000 and 2400 tokens, causal, Hq32/Hkv4/D128, fp32 out "
+                   f"[4,4400,{ncols}]")
     if "maxpool_cfg5" in per_op:
         nbytes = workloads.maxpool_bytes(c5["cu_q_cpu"], c5["cu_k_cpu"], [0], 2,
                                          -(-c5["max_context_len"] // 64))
@@ -613,7 +667,10 @@ def main():
             ("stage2_cfg5", bt, 1, "cfg5 selection: T=4096, Hq32/Hkv2, top-64 blocks of 64 tokens, "
                                    "paged bf16 K/V [2112,64,2,128], bf16 out [4096,32,128]"),
             ("stage2_cfg4", c4["bt"], 64, "cfg4 selection: 64 sequences, Hq32/Hkv2, top-64, paged "
-                                         "bf16 K/V [65536,64,2,128], bf16 out")):
+                                         "bf16 K/V [65536,64,2,128], bf16 out"),
+            ("stage2_decode", cd["bt"], 64, "stage1_decode's selection: 64 sequences of 1 token, "
+                                            "Hq32/Hkv2, top-64, paged bf16 K/V [65536,64,2,128], "
+                                            "bf16 out")):
         if name in per_op:
             nbytes, flop, n_ent = workloads.sparse_attn_work(b["topk_idx"], b["token_to_bs"],
                                                              b["token_pos_in_bs"], b["seqlen_q"],
@@ -629,10 +686,10 @@ def main():
                                             "gathered_gbs may exceed the HBM peak; beside it "
                                             "the same rows read with no arithmetic, "
                                             "stage2_gather_*)")
-            floor = name.replace("stage2_", "stage2_gather_")
-            if floor in per_op:
-                comps[name].update(gather_floor_us=per_op[floor] * 1e3,
-                                   frac_of_gather_floor=per_op[floor] / per_op[name])
+            gather = name.replace("stage2_", "stage2_gather_")
+            if gather in per_op:
+                comps[name].update(gather_us=per_op[gather] * 1e3,
+                                   gather_over_time=per_op[gather] / per_op[name])
     for name in ("stage2_gather_cfg5", "stage2_gather_cfg4"):
         if name in per_op:
             comps[name] = dict(us=per_op[name] * 1e3,
