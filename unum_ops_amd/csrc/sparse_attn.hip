@@ -224,7 +224,9 @@ __host__ __device__ constexpr int sa_swz(int key) {
   return (((key & 7) ^ (4 * ((key >> 3) & 1))) << 1) | ((key >> 3) & 1);
 }
 constexpr bool sa_lds_free() {
-  struct K { constexpr int operator()(int lane) const { return 16 * (lane & 15) + ((lane >> 4) ^ sa_swz(lane & 15)); } };
+  struct K {
+    constexpr int operator()(int lane) const { return 16 * (lane & 15) + ((lane >> 4) ^ sa_swz(lane & 15)); }
+  };
   if (!lds_b128_free(K{})) return false;
   for (int g = 0; g < 4; g += 2) {  // V: 32 lanes, eight keys, a chunk pair of each
     uint32_t pairs = 0;
@@ -686,7 +688,8 @@ __global__ __launch_bounds__(kWave* kSplit, 2) void sparse_attn_kernel(SaArgs a)
     // w + kSplit, ... of all of them.
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt) *reinterpret_cast<f32x4*>(slot + 1024 * dt + 16 * lane) = o[0][dt];
-    if (g == 0) *reinterpret_cast<float2*>(slot + 8192 + 8 * s) = make_float2(seen != 0 ? m_run[0] : -INFINITY, l_tot);
+    if (g == 0)
+      *reinterpret_cast<float2*>(slot + 8192 + 8 * s) = make_float2(seen != 0 ? m_run[0] : -INFINITY, l_tot);
     __syncthreads();
     float m[kSplit], l = 0.f, top = -3.402823466e38f;
     bool any = false;
